@@ -368,22 +368,24 @@ __device__ __forceinline__ void p0_tile_mixed(Args& A, const int2 tile, int symm
   }
 }
 
-// Helmholtz tiles of very far cell pairs in phase tier 2, from power sums of sigma = kappa^2 s / 2 (s =
-// r^2 - R^2) instead of point-pair kernel values. With R' = kappa R and u = 1 / R',
-//   e^{i (r' - R')} / r' = u sum_n H_n (-u sigma)^n / n!,  H_0 = 1, H_1 = u - i,
-//   H_{n+1} = (2n + 1) u H_n - H_{n-1}
-// (r'^2 = R'^2 + 2 sigma, d/d sigma = (1/r') d/dr', and (1/x d/dx)^n h_0(x) = (-1)^n h_n(x) / x^n for the
-// spherical Hankel functions, H_n = i e^{-iR'} R' h_n(R')), and the double-layer kernels'
-// e^{i(r'-R')} (1 - i r') / r'^3 is u^2 sum_n H_{n+1} (-u sigma)^n / n!: a cell pair needs
-// sum w w sigma^n, n = 1..6 (times the normal product), ten FP32 instructions a point
-// pair, independent of each other (two for sigma, two products, six sums), where rsq, the Newton
-// step and sine/cosine take a serial sixteen and a transcendental. Both rules in orbit form:
+// Helmholtz tiles of very far cell pairs in phase tier 2, from power sums of rho = mu s / (2 R) (s = r^2 -
+// R^2, mu = max(kappa, 1/R)) instead of point-pair kernel values. With a = 1 / (mu R), b = kappa / mu,
+//   e^{i kappa (r - R)} / r = (1/R) sum_n H_n (-rho)^n / n!,  H_0 = 1, H_1 = a - i b,
+//   H_{n+1} = (2n + 1) a H_n - b^2 H_{n-1}
+// (with x = kappa r and sigma = kappa^2 s / 2: x^2 = (kappa R)^2 + 2 sigma, d/d sigma = (1/x) d/dx, and
+// (1/x d/dx)^n h_0(x) = (-1)^n h_n(x) / x^n for the spherical Hankel functions; H_n = i e^{-i kappa R}
+// kappa R h_n(kappa R) (kappa / mu)^n), and the double-layer kernels' e^{i kappa (r - R)} (1 - i kappa r) /
+// r^3 is (mu / R^2) sum_n H_{n+1} (-rho)^n / n!. a and b are at most 1 and rho is small wherever kappa R
+// lies, so FP32 holds every factor: in powers of 1 / (kappa R) and sigma they overflow and underflow against each
+// other below kappa R ~ 1e-4. A cell pair needs sum w w rho^n, n = 1..6 (times the normal product), ten
+// FP32 instructions a point pair, independent of each other (two for rho, two products, six sums), where rsq,
+// the Newton step and sine/cosine take a serial sixteen and a transcendental. Both rules in orbit form:
 // x_p - c = tau d'_k, y_q - c = t d_k',
-//   sigma = (tau F_k + tau^2 g'_k) + t^2 g_k' + t (E_k' + tau N_kk').
-// Truncation, with |sigma u| <= 0.25 (tier 2) and |sigma u^2| <= 0.05 (t (rad_i + rad_j) / R for the
+//   rho = (tau F_k + tau^2 g'_k) + t^2 g_k' + t (E_k' + tau N_kk').
+// Truncation, with |rho| <= 0.25 where kappa R >= 1 (tier 2) and |a rho| <= 0.05 (t (rad_i + rad_j) / R for the
 // compiled rules' largest point radius t <= 0.7254): below 0.25^7 / 7! + 27 * 0.05^7 = 3e-8 of the
 // kernel value at the one extreme point pair, far less in the sum. Helmholtz, 20480 cells, k = 5,
-// complex64, whole assembly: single layer 4.12 -> 3.35 ms, relative error 5.2e-8 -> 4.9e-8; double
+// complex64, whole assembly: single layer 4.12 -> 3.36 ms, relative error 5.2e-8 -> 4.8e-8; double
 // layer 10.9 -> 7.35 ms, 9.6e-8 -> 5.7e-8.
 template <int Q, int OP, int CH = kChunk, int NW = 4, typename Args>
 __device__ __forceinline__ void p0_tile_moments(Args& A, const int2 tile, int symmetric,
@@ -395,12 +397,11 @@ __device__ __forceinline__ void p0_tile_moments(Args& A, const int2 tile, int sy
   const int i = tile.x * kTile + lane;
   const bool i_ok = i < A.n_test;
   const int il = i_ok ? i : A.n_test - 1;
-  const double kappa = fabs(A.k), kappa_inv = 1.0 / kappa;
-  const float sig = (float)(0.5 * kappa * kappa);
+  const double kappa = fabs(A.k);
   const float4* vtx32 = (const float4*)A.trial_vtx32;  // one grid: the test cells' records too
   const float4 te0 = vtx32[3 * (size_t)il], te1 = vtx32[3 * (size_t)il + 1], te2 = vtx32[3 * (size_t)il + 2];
   const float td[2][3] = {{te0.x, te0.y, te0.z}, {te1.x, te1.y, te1.z}};
-  const float tg[3] = {sig * te0.w, sig * te1.w, sig * te2.w};
+  const float tg[3] = {te0.w, te1.w, te2.w};
   // class weights divided by their sum over the points: M_0 = 1 exactly (with the normal products: D.n,
   // as each class's offsets from the centroid add up to zero), and the factor W (both cells' weight
   // sums) is applied in FP64; a rounding of M_0 would be common to all of v
@@ -446,8 +447,9 @@ __device__ __forceinline__ void p0_tile_moments(Args& A, const int2 tile, int sy
       const double Dx = ct[0] - sg[kGeoCentroid], Dy = ct[1] - sg[kGeoCentroid + 1], Dz = ct[2] - sg[kGeoCentroid + 2];
       const double R2 = fma(Dx, Dx, fma(Dy, Dy, Dz * Dz));
       const double Ri = rsqrt_fast(R2), R = R2 * Ri;
-      const double u64 = Ri * kappa_inv;
-      const float u = (float)u64;
+      const double mu = fmax(kappa, Ri);
+      const float sig = (float)(0.5 * mu * Ri);  // rho = sig s
+      const float a = (float)Ri * __builtin_amdgcn_rcpf((float)mu), b = (float)kappa * __builtin_amdgcn_rcpf((float)mu);
       const float D[3] = {2.0f * sig * (float)Dx, 2.0f * sig * (float)Dy, 2.0f * sig * (float)Dz};
       float E[3], F[3], N[3][3];
 #pragma unroll
@@ -480,7 +482,7 @@ __device__ __forceinline__ void p0_tile_moments(Args& A, const int2 tile, int sy
         }
         dnk[2] = -(dnk[0] + dnk[1]);
       }
-      float cq[Q];  // sigma's t^2 |d_k|^2
+      float cq[Q];  // rho's t^2 |d_k|^2
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
         const float t = orbit_t(Q, q);
@@ -498,13 +500,13 @@ __device__ __forceinline__ void p0_tile_moments(Args& A, const int2 tile, int sy
           for (int n = 1; n <= kOrder; ++n) m[b][n] = 0.0f;
 #pragma unroll
         for (int k = 0; k < decltype(npts)::value; ++k) {
-          const float a = fmaf(tau, F[k], (tau * tau) * tg[k]);
+          const float ap = fmaf(tau, F[k], (tau * tau * sig) * tg[k]);
           const float wk[3] = {fmaf(tau, N[k][0], E[0]), fmaf(tau, N[k][1], E[1]), fmaf(tau, N[k][2], E[2])};
           [[maybe_unused]] const float dnp = OP == 1 ? fmaf(tau, dnk[k], Dn) : Dn;
 #pragma unroll
           for (int q = 0; q < Q; ++q) {
             const float t = orbit_t(Q, q);
-            const float s = t == 0.0f ? a : fmaf(t, wk[orbit_vertex(Q, q)], a + cq[q]);
+            const float s = t == 0.0f ? ap : fmaf(t, wk[orbit_vertex(Q, q)], ap + cq[q]);
             float(&x)[kOrder + 1] = m[weight_class(Q, q)];
             const float s2 = s * s;
             if constexpr (kDN) {
@@ -540,33 +542,34 @@ __device__ __forceinline__ void p0_tile_moments(Args& A, const int2 tile, int sy
       for (int e = 0; e < n3; ++e)  // the body (18 point pairs) once for both classes: fewer registers
         test_class(e == 0 ? (float)orbit_t(Q, class_point(Q, c0)) : (float)orbit_t(Q, class_point(Q, NC - 1)),
                    e == 0 ? wt[c0] : wt[NC - 1], std::integral_constant<int, 3>{});
-      // sum_n H_n v_n (SL, HS) or H_{n+1} v_n (DL, ADL), v_n = M_n (-u)^n / n!; DL, ADL: n >= 1 here
-      cplxf h0 = {1.0f, 0.0f}, h1 = {u, -1.0f}, sum = {kDN ? 0.0f : 1.0f, 0.0f};
+      // sum_n H_n v_n (SL, HS) or H_{n+1} v_n (DL, ADL), v_n = M_n (-1)^n / n!; DL, ADL: n >= 1 here
+      cplxf h0 = {1.0f, 0.0f}, h1 = {a, -b}, sum = {kDN ? 0.0f : 1.0f, 0.0f};
+      const float b2 = b * b;
       float scale = 1.0f;
 #pragma unroll
       for (int n = 1; n <= kOrder; ++n) {
-        const float hc = (float)(2 * n + 1) * u;
-        const cplxf h2 = {fmaf(hc, h1.re, -h0.re), fmaf(hc, h1.im, -h0.im)};  // H_{n+1}
-        scale *= -u * (1.0f / (float)n);
+        const float hc = (float)(2 * n + 1) * a;
+        const cplxf h2 = {fmaf(hc, h1.re, -b2 * h0.re), fmaf(hc, h1.im, -b2 * h0.im)};  // H_{n+1}
+        scale *= -1.0f / (float)n;
         const float v = M[n] * scale;
         sum.re = fmaf(kDN ? h2.re : h1.re, v, sum.re);
         sum.im = fmaf(kDN ? h2.im : h1.im, v, sum.im);
         h0 = h1;
         h1 = h2;
       }
-      // k < 0 (conjugate), rotation by e^{ikR} as p0_tile_mixed; the factor kappa u = 1 / R (kappa^3 u^2)
-      // and H_1 M_0 of the double layers in FP64, as their FP32 roundings would be common to the whole sum
+      // k < 0 (conjugate), rotation by e^{ikR} as p0_tile_mixed; the factor 1 / R (1 / R^2) and mu H_1 M_0
+      // of the double layers in FP64, as their FP32 roundings would be common to the whole sum
       const double kR = A.k * R;
       const double nr = rint(kR * 0.63661977236758134);
       const double tr = fma(-nr, 6.123233995736766e-17, fma(-nr, 1.5707963267948966, kR));
       float sn, cs;
       sincos_f32_quadrant((float)tr, (int)nr, &sn, &cs);
       double f = kInv4Pi * Ri * (0.25 * tgeo[12] * sg[12]);
-      if constexpr (kDN) f *= kappa * Ri;
+      if constexpr (kDN) f *= Ri;
       if constexpr (OP == 3) f *= -A.k * A.k * (nx[0] * sg[9] + nx[1] * sg[10] + nx[2] * sg[11]);
       cplx v;
       if constexpr (kDN) {
-        const double re = fma(dn64, u64, (double)sum.re), im0 = (double)sum.im - dn64;
+        const double re = fma(dn64, Ri, mu * (double)sum.re), im0 = fma(mu, (double)sum.im, -(kappa * dn64));
         const double im = A.k < 0.0 ? -im0 : im0;
         v = {(re * cs - im * sn) * f, (re * sn + im * cs) * f};
       } else {

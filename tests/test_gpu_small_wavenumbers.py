@@ -1,0 +1,49 @@
+"""Helmholtz operators at small wavenumbers, where quantities scaled by |k| leave their type's range:
+mixed precision (single and batched) against FP64, all operators: 1e-6 relative in the norm as for
+every mixed-precision operator, all entries finite."""
+import numpy as np
+import pytest
+import torch
+
+from bempp_amd.assembly.batch import BatchAssembler
+from bempp_amd.assembly.boundary import (BoundaryAssemblerOptions, OperatorType, Precision, create_helmholtz_assembler)
+from bempp_amd.element import Continuity, Family, ReferenceCellType, create_family
+from bempp_amd.function_space import function_space
+from bempp_amd.grid import Grid
+from test_gpu_tile_parts import _torus
+
+pytestmark = pytest.mark.gpu
+
+
+def _options(nq=6, precision=Precision.FP64):
+    o = BoundaryAssemblerOptions()
+    o.set_regular_quadrature_degree(ReferenceCellType.Triangle, nq)
+    o.set_precision(precision)
+    return o
+
+
+def _space(g, degree, continuity=Continuity.Standard):
+    return function_space(g, create_family(Family.Lagrange, degree, continuity if degree else Continuity.Discontinuous))
+
+
+def _thin_torus():
+    """2304 cells in 36 tiles, most of them very far from each other (tube radius 0.1)."""
+    p, c = _torus(96, 12)
+    ring = p * [1, 1, 0]
+    ring /= np.linalg.norm(ring, axis=1, keepdims=True)
+    return ring + 0.25 * (p - ring), c
+
+
+@pytest.mark.parametrize("k", [1e-2, 1e-3, -1e-4, 1e-5, 1e-6, 1e-8, 1e-12])
+@pytest.mark.parametrize("op", list(OperatorType)[:4])
+@pytest.mark.parametrize("nq", [6, 7])
+def test_mixed(k, op, nq):
+    p, c = _thin_torus()
+    s = _space(Grid(p, c), 0)
+    R = create_helmholtz_assembler(k, op, _options(nq)).assemble_device(s, s)
+    a = [create_helmholtz_assembler(x, op, _options(nq, Precision.Mixed)) for x in (k, 2.0 * k)]
+    A = a[0].assemble_device(s, s)
+    B = BatchAssembler(a, [s, s]).assemble()[0]
+    for x in (A, B):
+        assert torch.isfinite(torch.view_as_real(x)).all()
+        assert torch.linalg.norm(x - R) <= 1e-6 * torch.linalg.norm(R)
