@@ -41,6 +41,7 @@ struct DeviceGridCache {
   int4* pairs = nullptr;          // adjacent pairs
   int npairs = -1;
   double max_radius = 0.0;        // largest centroid-to-vertex distance of any cell
+  double min_radius = 0.0;        // smallest of the cells' radii
   double max_edge = 0.0;          // longest edge of any cell
   std::map<int, float*> pts32;    // regular point count -> [nc][Q][4] FP32 offsets from the centroid, w*jdet
   std::map<int, float*> vtx32;    // regular point count -> [nc][3][4] FP32 vertex offsets, class weights
@@ -201,11 +202,12 @@ DeviceGridCache* grid_cache(Grid& g, int device) {
   if (c && c->geo) return c;
   const int64_t nc = g.nc();
   std::vector<double> geo(nc * dev::kGeoStride);
-  double max_radius = 0.0, max_edge = 0.0;
+  double max_radius = 0.0, min_radius = INFINITY, max_edge = 0.0;
   for (int64_t i = 0; i < nc; ++i) {
     double* r = &geo[i * dev::kGeoStride];
     cell_record(g, i, r);
     max_radius = std::max(max_radius, r[dev::kGeoRadius]);
+    min_radius = std::min(min_radius, r[dev::kGeoRadius]);
     for (int m = 0; m < 3; ++m) {  // the J-scaled curls are the edge vectors
       const double* e = r + 13 + 3 * m;
       max_edge = std::max(max_edge, std::sqrt(e[0] * e[0] + e[1] * e[1] + e[2] * e[2]));
@@ -224,6 +226,7 @@ DeviceGridCache* grid_cache(Grid& g, int device) {
   }
   c->geo = upload(geo);
   c->max_radius = max_radius;
+  c->min_radius = min_radius;
   c->max_edge = max_edge;
   return c;
 }
@@ -986,7 +989,12 @@ Prepared prepare(const Assembler& a, const FunctionSpace& trial_c, const Functio
   // than the FP32 point pairs of the mixed tiles (FP32 without packed math issues at the
   // FP64 rate)
   const bool laplace_hs_p1 = a.kind == kLaplace && a.op == kHS && test.nb == 3 && trial.nb == 3 && R.orbit_form;
-  P.mixed = a.options.precision == kMixed && P.same_grid && compiled_q && !laplace_hs_p1;
+  // The FP32 point pairs of the Helmholtz tiles are in lengths scaled by |k|: (|k| r)^-3 overflows below
+  // |k| r = 1e-13 and |k|^3 underflows below |k| = 1e-13 (NaN from there on), so wavenumbers
+  // that near to zero (k = 0 itself runs the Laplace tiles) stay in FP64.
+  const double scaled = std::fabs(a.k) * std::min(1.0, tc->min_radius);
+  const bool too_small = a.kind == kHelmholtz && a.k != 0.0 && scaled < 1e-12;
+  P.mixed = a.options.precision == kMixed && P.same_grid && compiled_q && !laplace_hs_p1 && !too_small;
   P.near = nullptr;
   P.nnear = 0;
   P.near_segs = nullptr;

@@ -34,7 +34,7 @@ def _thin_torus():
     return ring + 0.25 * (p - ring), c
 
 
-@pytest.mark.parametrize("k", [1e-2, 1e-3, -1e-4, 1e-5, 1e-6, 1e-8, 1e-12])
+@pytest.mark.parametrize("k", [1e-2, 1e-3, -1e-4, 1e-5, 1e-6, 1e-8, 1e-12, 1e-20, 1e-40])
 @pytest.mark.parametrize("op", list(OperatorType)[:4])
 @pytest.mark.parametrize("nq", [6, 7])
 def test_mixed(k, op, nq):
