@@ -1015,7 +1015,7 @@ void assemble_cells_device(const Assembler& a, const FunctionSpace& trial, const
   // phase tier from the grid-wide bound on |k (r - R)| by the rule points' distances from their centroids, with a
   // margin for rounding (the tiers' polynomials hold to 0.25, 0.5 and 1.5 exactly)
   int tier = 0;
-  if (a.kind == kHelmholtz && a.k != 0.0) {
+  if (a.kind == kHelmholtz && dev::scalable(a.k, A.radius_sum)) {
     const double bound = std::fabs(a.k) * A.offset_sum * (1.0 + 1e-12);
     tier = bound <= 0.25 ? 2 : bound <= 0.5 ? 1 : bound <= 1.5 ? 3 : 0;
   }

@@ -952,9 +952,7 @@ Prepared prepare(const Assembler& a, const FunctionSpace& trial_c, const Functio
   // (bound 0.69) takes 0.62 ms in tier 3, 0.83 ms in tier 0
   const RuleGroups rg = rule_groups(P.Q);
   const double phase_bound = std::fabs(a.k) * rule_radius(rg) * (tc->max_radius + sc->max_radius) * (1.0 + 1e-12);
-  // (|k| below 1e-100, k = 0 included, takes the full reduction: the centred tile sums work
-  // in lengths scaled by |k|)
-  const bool centred = a.kind == kHelmholtz && std::fabs(a.k) >= 1e-100;
+  const bool centred = a.kind == kHelmholtz && dev::scalable(a.k, tc->max_radius + sc->max_radius);
   P.tier = !centred ? 0 : phase_bound <= 0.25 ? 2 : phase_bound <= 0.5 ? 1 : phase_bound <= 1.5 ? 3 : 0;
   // points of two cells sharing a vertex are at most two longest edges apart (each is within one
   // of the vertex)
@@ -1441,7 +1439,8 @@ PotentialInputs potential_inputs(const Assembler& a, const FunctionSpace& space_
   P.ncells = (int)grid.nc();
   P.nb = space.nb;
   P.ndofs = space.size;
-  P.max_radius = rule_radius(rg) * gc->max_radius;
+  P.max_radius = gc->max_radius;
+  P.rule_radius = rule_radius(rg);
   P.out_type = out_type(a.dtype);
   return P;
 }

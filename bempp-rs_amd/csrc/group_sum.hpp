@@ -76,6 +76,14 @@ __device__ __forceinline__ cplx group_kernel(double h, double dn, double kR, dou
   }
 }
 
+// Whether lengths can be scaled by |k| for cells of this radius (host): (kappa / 2)^2 r^2 must not
+// underflow, nor (4 / (kappa r))^3 and its factor (kappa / 4)^3 leave the range, with room for point pairs
+// much nearer than the radius. Other wavenumbers, k = 0 among them, take phase tier 0, which is unscaled.
+inline bool scalable(double k, double radius) {
+  const double kappa = k < 0.0 ? -k : k;
+  return kappa >= 1e-80 && kappa * radius >= 1e-80;
+}
+
 template <int OP, bool HELM, int TIER>
 __device__ __forceinline__ double group_factor(double kappa) {
   const double f = HELM && TIER > 0 ? 0.25 * kappa : 0.5;

@@ -1434,7 +1434,8 @@ struct PotentialInputs {
   int Q;
   int nb;
   int64_t ndofs;
-  double max_radius;       // largest distance of a rule point from its cell's centroid
+  double max_radius;       // largest centroid-to-vertex distance of any cell
+  double rule_radius;      // largest distance of a rule point from the centroid of a cell of radius 1
   int out_type;
 };
 PotentialInputs potential_inputs(const Assembler& a, const FunctionSpace& space, int64_t npoints, void* stream);

@@ -268,9 +268,9 @@ void assemble_potential_device(const Assembler& a, const FunctionSpace& space, c
   if (groups * P.parts > INT32_MAX) throw Error("too many evaluation points");
   const dim3 g((unsigned)(groups * P.parts));
   const bool helm = a.kind == kHelmholtz;
-  // |k (r - R)| <= |k| t rad (with a margin for the rounding of r and R); k = 0 is exact in any tier
-  const double bound = std::fabs(a.k) * in.max_radius * (1.0 + 1e-12);
-  const int tier = !helm ? 0 : bound <= 0.25 ? 2 : bound <= 0.5 ? 1 : bound <= 1.5 ? 3 : 0;
+  // |k (r - R)| <= |k| t rad (with a margin for the rounding of r and R)
+  const double bound = std::fabs(a.k) * in.rule_radius * in.max_radius * (1.0 + 1e-12);
+  const int tier = !helm || !dev::scalable(a.k, in.max_radius) ? 0 : bound <= 0.25 ? 2 : bound <= 0.5 ? 1 : bound <= 1.5 ? 3 : 0;
   if (a.op == kSL) launch_potential<0>(in.Q, helm, tier, in.nb, g, s, P);
   else launch_potential<1>(in.Q, helm, tier, in.nb, g, s, P);
   HIP_CHECK_P(hipGetLastError());
