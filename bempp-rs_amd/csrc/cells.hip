@@ -51,7 +51,7 @@ struct CellsArgs {
   const double* srec;
   // P0 single layer: the test points again as [point of the cell][cell][4] (a wavefront's 64 test
   // cells read consecutive memory), and the trial points relative to their cells' centroids,
-  // [points][kSlRec]: offset (3), its square, w J, pad
+  // [points][kSlRec]: offset (3), its square, w J, the cell's radius
   const double* txt;
   const double* sxo;
   const int* tfirst;   // first record of each test cell [n_test + 1]
@@ -351,6 +351,17 @@ __global__ void __launch_bounds__(256) cells_regular_kernel(const CellsArgs A) {
 
 constexpr int kSlRec = 6;
 
+// Largest distance of a vertex from the centroid (cv: as cell_centroid).
+template <typename V>
+__device__ __forceinline__ double cell_radius(const V& cv, bool quad, const double (&cen)[3]) {
+  double m = 0.0;
+  for (int v = 0; v < (quad ? 4 : 3); ++v) {
+    const double x = cv[3 * v] - cen[0], y = cv[3 * v + 1] - cen[1], z = cv[3 * v + 2] - cen[2];
+    m = fmax(m, x * x + y * y + z * z);
+  }
+  return sqrt(m);
+}
+
 // The compact views of the point records (CellsArgs: txw, txt, sxo): a thread per point of a cell,
 // padded to the largest cell's count (txt is zero there). Made on the device, where they would
 // otherwise be filled on the host and uploaded: 86400 points (5400 cells), a new grid's first call
@@ -377,7 +388,7 @@ __global__ void __launch_bounds__(256) point_views_kernel(const double* __restri
   }
   v[3] = s;
   v[4] = x[3];
-  v[5] = 0.0;
+  v[5] = cell_radius(cv + 12 * (size_t)c, vid[4 * (size_t)c + 3] >= 0, cen);
   for (int m = 0; m < 4; ++m) o[m] = xw[4 * (size_t)r + m] = x[m];
 }
 
@@ -385,7 +396,8 @@ __global__ void __launch_bounds__(256) point_views_kernel(const double* __restri
 // centroid) r^2 = |X|^2 + |o_q|^2 - 2 X.o_q: four FMAs per point pair instead of the seven
 // instructions of a difference, its square and the length scaling; four test points at a time
 // share each trial point read from LDS (broadcasts; 48-byte records, so that a barrier covers
-// 32 cells of 16 points), and the test points are read coalesced.
+// 32 cells of 16 points), and the test points are read coalesced. Cells near each other take r^2 from
+// the differences X - o_q (group_near).
 // Bound by FP64 VALU issue, 22 + rsq (Helmholtz tier 2) instructions per point pair.
 // Helmholtz, 5400 cells of 16 points, tier 1, with the adjacent pairs: 4.94 -> 4.58 ms.
 constexpr int kSlStage = 512;  // records staged per workgroup (24 KB)
@@ -402,6 +414,7 @@ __global__ void __launch_bounds__(256) cells_sl_p0_kernel(const CellsArgs A) {
   for (int m = 0; m < 4; ++m) tv[m] = A.tvid[4 * il + m];
   double ct[3];
   cell_centroid(A.tcv + 12 * (size_t)il, tv[3] >= 0, ct);
+  const double trad = cell_radius(A.tcv + 12 * (size_t)il, tv[3] >= 0, ct);
   const int np = A.tfirst[il + 1] - A.tfirst[il];
   const auto scv = constant_view(A.scv);
   const auto svid = constant_view(A.svid);
@@ -430,35 +443,47 @@ __global__ void __launch_bounds__(256) cells_sl_p0_kernel(const CellsArgs A) {
     cplx e = {1.0, 0.0};
     if constexpr (TIER > 0) e = pair_phase(ct, cs, kappa, &kR);
     cplx sum = {0.0, 0.0};
-    for (int p = 0; p < np; p += PP) {
-      double base[PP], U[PP][3], w[PP];
-      cplx acc[PP];
-#pragma unroll
-      for (int u = 0; u < PP; ++u) {
-        // past the cell's last point: the last one again, with weight 0
-        const double4 x = ((const double4*)A.txt)[(size_t)min(p + u, np - 1) * A.n_test + il];
-        const double X[3] = {x.x - cs[0], x.y - cs[1], x.z - cs[2]};
-        w[u] = p + u < np ? x.w : 0.0;
-        base[u] = sc * (X[0] * X[0] + X[1] * X[1] + X[2] * X[2]);
-#pragma unroll
-        for (int d = 0; d < 3; ++d) U[u][d] = -2.0 * sc * X[d];
-        acc[u] = {0.0, 0.0};
-      }
-#pragma unroll 1
-      for (int q = 0; q < nq; ++q) {
-        const double* Q = Qj + q * kSlRec;
-        const double o0 = Q[0], o1 = Q[1], o2 = Q[2], g = sc * Q[3], wq = Q[4];
+    auto point_pairs = [&](auto by_differences) {
+      constexpr bool NEAR = decltype(by_differences)::value;
+      for (int p = 0; p < np; p += PP) {
+        double base[PP], U[PP][3], w[PP];  // NEAR: U = X
+        cplx acc[PP];
 #pragma unroll
         for (int u = 0; u < PP; ++u) {
-          const double h = fma(o0, U[u][0], fma(o1, U[u][1], fma(o2, U[u][2], g + base[u])));
-          const cplx v = group_kernel<0, HELM, TIER>(h, 0.0, kR, khalf);
-          acc[u].re = fma(v.re, wq, acc[u].re);
-          acc[u].im = fma(v.im, wq, acc[u].im);
-        }
-      }
+          // past the cell's last point: the last one again, with weight 0
+          const double4 x = ((const double4*)A.txt)[(size_t)min(p + u, np - 1) * A.n_test + il];
+          const double X[3] = {x.x - cs[0], x.y - cs[1], x.z - cs[2]};
+          w[u] = p + u < np ? x.w : 0.0;
+          base[u] = sc * (X[0] * X[0] + X[1] * X[1] + X[2] * X[2]);
 #pragma unroll
-      for (int u = 0; u < PP; ++u) add_scaled(sum, acc[u], w[u]);
-    }
+          for (int d = 0; d < 3; ++d) U[u][d] = NEAR ? X[d] : -2.0 * sc * X[d];
+          acc[u] = {0.0, 0.0};
+        }
+#pragma unroll 1
+        for (int q = 0; q < nq; ++q) {
+          const double* Q = Qj + q * kSlRec;
+          const double o0 = Q[0], o1 = Q[1], o2 = Q[2], g = sc * Q[3], wq = Q[4];
+#pragma unroll
+          for (int u = 0; u < PP; ++u) {
+            double h;
+            if constexpr (NEAR) {
+              const double x = U[u][0] - o0, y = U[u][1] - o1, z = U[u][2] - o2;
+              h = sc * (x * x + y * y + z * z);
+            } else {
+              h = fma(o0, U[u][0], fma(o1, U[u][1], fma(o2, U[u][2], g + base[u])));
+            }
+            const cplx v = group_kernel<0, HELM, TIER>(h, 0.0, kR, khalf);
+            acc[u].re = fma(v.re, wq, acc[u].re);
+            acc[u].im = fma(v.im, wq, acc[u].im);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < PP; ++u) add_scaled(sum, acc[u], w[u]);
+      }
+    };
+    const double X = ct[0] - cs[0], Y = ct[1] - cs[1], Z = ct[2] - cs[2];
+    if (__any(group_near(X * X + Y * Y + Z * Z, trad + Qj[5]))) point_pairs(std::true_type{});  // uniform
+    else point_pairs(std::false_type{});
     const double f = group_factor<0, HELM, TIER>(kappa) * kInv4Pi;
     cplx v = {sum.re * f, sum.im * f};
     if constexpr (TIER > 0) v = cmul(v, e);

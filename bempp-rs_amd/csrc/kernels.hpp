@@ -394,6 +394,7 @@ struct P1TestCell {
   double td[2][3];  // vertex offsets from the centroid
   double nx[3], ct[3];
   double jx;
+  float rad;
   // hypersingular: the J-scaled surface curls of basis functions 1, 2, in LDS at [6][64] (a
   // tile's wavefronts share its test cells; in registers they would cost a wave per SIMD)
   const double* curl;
@@ -419,14 +420,24 @@ __device__ __forceinline__ P1TestCell<OP> p1_test_cell(const RegularArgs& A, int
   }
   t.curl = lds + (threadIdx.x & 63);
   t.jx = geo[12];
+  t.rad = (float)geo[kGeoRadius];
   return t;
 }
 
-// The local block of a regular cell pair with a P1 side, in group form (group_sum.hpp): the lane's
-// test cell t and the wave-uniform trial cell j; add(a, b, value) for each entry. The
+// Whether the lane's test cell t and trial cell j are near (group_near).
+template <int OP>
+__device__ __forceinline__ bool p1_near(const RegularArgs& A, const P1TestCell<OP>& t, int j) {
+  const auto sg = constant_view(A.trial_geo) + (size_t)j * kGeoStride;
+  const double D[3] = {t.ct[0] - sg[kGeoCentroid], t.ct[1] - sg[kGeoCentroid + 1], t.ct[2] - sg[kGeoCentroid + 2]};
+  return group_near(D[0] * D[0] + D[1] * D[1] + D[2] * D[2], t.rad + sg[kGeoRadius]);
+}
+
+// The local block of a regular cell pair with a P1 side, in group form or, NEAR, from differences
+// (group_sum.hpp): the lane's test cell t and the trial cell j, wave-uniform (NEAR: the lane's); add(a, b, value)
+// for each entry. The
 // hypersingular entries are (curl_a . curl_b) sum(K) - k^2 n_x.n_y M_ab with the Jacobians of
 // the curls and of the weights cancelling in the first term; the Laplace one needs only the sum.
-template <int Q, int OP, bool HELM, int TIER, typename Add>
+template <int Q, int OP, bool HELM, int TIER, bool NEAR, typename Add>
 __device__ __forceinline__ void p1_cell_pair(const RegularArgs& A, const P1TestCell<OP>& t, int j, Add add) {
   constexpr bool SUM = OP == 3 && !HELM;
   constexpr int NB = SUM ? 1 : 3;
@@ -436,18 +447,23 @@ __device__ __forceinline__ void p1_cell_pair(const RegularArgs& A, const P1TestC
   const double g[3] = {sv[3], sv[7], sv[11]};
   const double ny[3] = {sg[9], sg[10], sg[11]};
   const double D[3] = {t.ct[0] - sg[kGeoCentroid], t.ct[1] - sg[kGeoCentroid + 1], t.ct[2] - sg[kGeoCentroid + 2]};
+  const double R2 = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
   const double kappa = HELM ? fabs(A.k) : 0.0;
   double kR = 0.0;
   cplx e = {1.0, 0.0};
   if constexpr (TIER > 0) {
-    const double R2 = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
     kR = kappa * (R2 * rsqrt_nr(R2));
     sincos_cw(kR, &e.im, &e.re);
   }
   cplx M[NB][NB];
-  group_pair_sum<Q, OP, HELM, TIER, !SUM>(A, t.td, D, t.nx, ny, d, g, constant_view(A.trial_gq) + (size_t)j * 3 * A.ngroups,
-                                          kappa, kR, M);
-  const double f = group_factor<OP, HELM, TIER>(kappa) * kInv4Pi * (OP == 3 ? 1.0 : t.jx * sg[12]);
+  double f = kInv4Pi * (OP == 3 ? 1.0 : t.jx * sg[12]);
+  if constexpr (NEAR) {
+    near_pair_sum<OP, HELM, TIER, !SUM>(A, t.td, D, t.nx, ny, d, kappa, kR, M);
+  } else {
+    group_pair_sum<Q, OP, HELM, TIER, !SUM>(A, t.td, D, t.nx, ny, d, g, constant_view(A.trial_gq) + (size_t)j * 3 * A.ngroups,
+                                            kappa, kR, M);
+    f *= group_factor<OP, HELM, TIER>(kappa);
+  }
   e = {e.re * f, e.im * f};
   const double sgn = HELM && A.k < 0.0 ? -1.0 : 1.0;  // e^{-i kappa r} is the conjugate
   cplx sum = {0.0, 0.0};
@@ -510,23 +526,33 @@ __global__ void __launch_bounds__(256) regular_kernel(const RegularArgs A) {
   const auto trial_vid = constant_view(A.trial_vid);
   const int j0 = blockIdx.y * A.trial_chunk;
   const int j1 = min(j0 + A.trial_chunk, A.n_trial);
-  for (int j = j0; j < j1; ++j) {
-    const int sv0 = trial_vid[4 * j], sv1 = trial_vid[4 * j + 1], sv2 = trial_vid[4 * j + 2];
-    const bool adjacent = A.same_grid && (tv0 == sv0 || tv0 == sv1 || tv0 == sv2 || tv1 == sv0 || tv1 == sv1 ||
-                                          tv1 == sv2 || tv2 == sv0 || tv2 == sv1 || tv2 == sv2);
-    if (!i_ok) continue;
-    const auto store = [&](int a, int b, cplx v) {
+  for (int jb = j0; jb < j1; jb += 32) {
+    unsigned near = 0;  // the lane's near trial cells from jb on
+    const auto store = [&](int j, int a, int b, cplx v) {
       const long long col = A.trial_dofs[(size_t)j * A.nbs + b];
       const long long row = A.test_dofs[(size_t)i * A.nbt + a];
       store_value(A.out, row + A.ld * col, v, A.out_type, A.mode);
     };
-    if (adjacent) {
-      if (A.mode == kStore)
-        for (int b = 0; b < A.nbs; ++b)
-          for (int a = 0; a < A.nbt; ++a) store(a, b, cplx{0.0, 0.0});
-      continue;
+    for (int j = jb; j < min(jb + 32, j1); ++j) {
+      const int sv0 = trial_vid[4 * j], sv1 = trial_vid[4 * j + 1], sv2 = trial_vid[4 * j + 2];
+      const bool adjacent = A.same_grid && (tv0 == sv0 || tv0 == sv1 || tv0 == sv2 || tv1 == sv0 || tv1 == sv1 ||
+                                            tv1 == sv2 || tv2 == sv0 || tv2 == sv1 || tv2 == sv2);
+      if (!i_ok) continue;
+      if (adjacent) {
+        if (A.mode == kStore)
+          for (int b = 0; b < A.nbs; ++b)
+            for (int a = 0; a < A.nbt; ++a) store(j, a, b, cplx{0.0, 0.0});
+        continue;
+      }
+      if (p1_near(A, t, j))
+        near |= 1u << (j - jb);
+      else
+        p1_cell_pair<Q, OP, HELM, CENTRED, false>(A, t, j, [&](int a, int b, cplx v) { store(j, a, b, v); });
     }
-    p1_cell_pair<Q, OP, HELM, CENTRED>(A, t, j, store);
+    for (; near != 0; near &= near - 1) {
+      const int j = jb + __ffs(near) - 1;
+      p1_cell_pair<Q, OP, HELM, CENTRED, true>(A, t, j, [&](int a, int b, cplx v) { store(j, a, b, v); });
+    }
   }
 }
 
@@ -845,18 +871,27 @@ regular_tiled_lds(const RegularArgs A, const int2* __restrict__ tiles, int symme
   const auto trial_vid = constant_view(A.trial_vid);
   const auto trial_ldof = constant_view(A.trial_ldof);
   const int tpw = kTile / 4 / split;  // trial cells per wavefront
+  const int jw = tile.y * kTile + (part * 4 + wave) * tpw;
+  unsigned near = 0;  // the lane's near trial cells from jw on
+  const auto add = [&](int j, int a, int b, cplx v) {
+    const int ls = trial_ldof[(size_t)j * A.nbs + b];
+    tile_add<HELM>(tile_acc, nacc, ls * ndt + lt[a], v);
+  };
 #pragma unroll 1
-  for (int jj = 0; jj < tpw; ++jj) {
-    const int j = tile.y * kTile + (part * 4 + wave) * tpw + jj;
-    if (j >= A.n_trial) break;  // wave-uniform
+  for (int j = jw; j < min(jw + tpw, A.n_trial); ++j) {
     const int sv0 = trial_vid[4 * j], sv1 = trial_vid[4 * j + 1], sv2 = trial_vid[4 * j + 2];
     const bool adjacent = A.same_grid && (tv0 == sv0 || tv0 == sv1 || tv0 == sv2 || tv1 == sv0 || tv1 == sv1 ||
                                           tv1 == sv2 || tv2 == sv0 || tv2 == sv1 || tv2 == sv2);
     if (adjacent || !i_ok) continue;
-    p1_cell_pair<Q, OP, HELM, CENTRED>(A, t, j, [&](int a, int b, cplx v) {
-      const int ls = trial_ldof[(size_t)j * A.nbs + b];
-      tile_add<HELM>(tile_acc, nacc, ls * ndt + lt[a], v);
-    });
+    if (p1_near(A, t, j))
+      near |= 1u << (j - jw);
+    else
+      p1_cell_pair<Q, OP, HELM, CENTRED, false>(A, t, j, [&](int a, int b, cplx v) { add(j, a, b, v); });
+  }
+#pragma unroll 1
+  for (; near != 0; near &= near - 1) {
+    const int j = jw + __ffs(near) - 1;
+    p1_cell_pair<Q, OP, HELM, CENTRED, true>(A, t, j, [&](int a, int b, cplx v) { add(j, a, b, v); });
   }
   __syncthreads();
   flush_tile<HELM>(A, tile_acc, t0, ndt, s0, nds, symmetric && tile.x != tile.y);
@@ -921,6 +956,7 @@ __device__ __forceinline__ void p0_tile(Args& A, const int2 tile, int symmetric,
   const double nx[3] = {tgeo[9], tgeo[10], tgeo[11]};
   const double ct[3] = {tgeo[kGeoCentroid], tgeo[kGeoCentroid + 1], tgeo[kGeoCentroid + 2]};
   const double tjx = tgeo[12];
+  [[maybe_unused]] const float trad = (float)tgeo[kGeoRadius];
   const int tv0 = A.test_vid[4 * il], tv1 = A.test_vid[4 * il + 1], tv2 = A.test_vid[4 * il + 2];
   const bool mirror = symmetric && tile.x != tile.y;
   const int skind = fast_store_kind(A.out_type, A.mode);
@@ -935,6 +971,33 @@ __device__ __forceinline__ void p0_tile(Args& A, const int2 tile, int symmetric,
   cplx yi = {0.0, 0.0};
   for (int c = 0; c < tpw; c += ch) {
     const int jbase = tile.y * kTile + (part * NW + wave) * tpw + c;
+    unsigned near = 0;  // the lane's near trial cells of the chunk (the orbit sums of the dense tiles take r^2 by terms at
+                        // any distance)
+    auto finish = [&](int jj, auto sg, cplx acc) {
+      const int j = jbase + jj;
+      if constexpr (OP == 3) {  // P0 hypersingular: only the Helmholtz -k^2 n_x.n_y term survives
+        const double nn = HELM ? -A.k * A.k * (nx[0] * sg[9] + nx[1] * sg[10] + nx[2] * sg[11]) : 0.0;
+        acc = {nn * acc.re, nn * acc.im};
+      }
+      // adjacent pairs get 0 here (their Duffy value is added by the singular kernel)
+      const cplx v = {acc.re * kInv4Pi, acc.im * kInv4Pi};
+      if constexpr (APPLY) {
+        const auto uj = constant_view(u) + 2 * (size_t)j;
+        const cplx t = cmul(v, {uj[0], uj[1]});
+        yi.re += t.re;
+        yi.im += t.im;
+      } else if (i_ok) {
+        store_entry(A.out, (long long)i + A.ld * (long long)j, v, skind, A.out_type, A.mode);
+      }
+      if (mirror) lds[wave][jj][lane] = make_double2(v.re, v.im);
+    };
+    // the sum of group_pair_sum or near_pair_sum, times f and e^{i kappa R}
+    auto scaled = [&](cplx m, double f, cplx e) {
+      cplx v = {m.re * f, m.im * f};
+      if constexpr (CENTRED) v = cmul(v, e);
+      if (HELM && A.k < 0.0) v.im = -v.im;
+      return v;
+    };
 #pragma unroll 1
     for (int jj = 0; jj < ch; ++jj) {
       const int j = jbase + jj;
@@ -952,25 +1015,27 @@ __device__ __forceinline__ void p0_tile(Args& A, const int2 tile, int symmetric,
       const bool adjacent = A.same_grid && (tv0 == sv0 || tv0 == sv1 || tv0 == sv2 || tv1 == sv0 || tv1 == sv1 ||
                                             tv1 == sv2 || tv2 == sv0 || tv2 == sv1 || tv2 == sv2);
       const double ny[3] = {sg[9], sg[10], sg[11]};
+      const double cs[3] = {sg[kGeoCentroid], sg[kGeoCentroid + 1], sg[kGeoCentroid + 2]};
+      const double D[3] = {ct[0] - cs[0], ct[1] - cs[1], ct[2] - cs[2]};
+      const double R2 = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
+      bool left = adjacent;  // to the singular kernel, or to the near pairs below
+      if constexpr (GEN || APPLY)
+        if (!adjacent && group_near(R2, trad + sg[kGeoRadius])) {
+          near |= 1u << jj;
+          left = true;
+        }
       cplx acc = {0.0, 0.0};
-      if (!adjacent) {
-        const double cs[3] = {sg[kGeoCentroid], sg[kGeoCentroid + 1], sg[kGeoCentroid + 2]};
-        const double D[3] = {ct[0] - cs[0], ct[1] - cs[1], ct[2] - cs[2]};
-        const double R2 = D[0] * D[0] + D[1] * D[1] + D[2] * D[2];
+      if (!left) {
         if constexpr (GEN) {
           const double kappa = HELM ? fabs(A.k) : 0.0;
           double kR = 0.0;
-          cplx e = {1.0, 0.0};
+          cplx e = {1.0, 0.0}, M[1][1];
           if constexpr (CENTRED) e = pair_phase(ct, cs, kappa, &kR);
           const double d[2][3] = {{sp[0], sp[1], sp[2]}, {sp[4], sp[5], sp[6]}};
           const double g[3] = {sp[3], sp[7], sp[11]};
-          cplx M[1][1];
           group_pair_sum<Q, OP, HELM, CENTRED, false>(A, td, D, nx, ny, d, g, trial_gq + (size_t)j * 3 * A.ngroups, kappa, kR,
                                                       M);
-          const double f = group_factor<OP, HELM, CENTRED>(kappa) * (tjx * sg[12]);
-          acc = {M[0][0].re * f, M[0][0].im * f};
-          if constexpr (CENTRED) acc = cmul(acc, e);
-          if (HELM && A.k < 0.0) acc.im = -acc.im;
+          acc = scaled(M[0][0], group_factor<OP, HELM, CENTRED>(kappa) * (tjx * sg[12]), e);
         } else if constexpr (CENTRED) {
           double kR;
           const cplx e = pair_phase(ct, cs, A.k, &kR);
@@ -979,22 +1044,26 @@ __device__ __forceinline__ void p0_tile(Args& A, const int2 tile, int symmetric,
           acc = p0_pair_orbit<Q, OP, HELM, 0>(td, tau2g, twc, sp, D, R2, nx, ny, A.k, 0.0);
         }
       }
-      if constexpr (OP == 3) {  // P0 hypersingular: only the Helmholtz -k^2 n_x.n_y term survives
-        const double nn = HELM ? -A.k * A.k * (nx[0] * ny[0] + nx[1] * ny[1] + nx[2] * ny[2]) : 0.0;
-        acc = {nn * acc.re, nn * acc.im};
-      }
-      // adjacent pairs get 0 here (their Duffy value is added by the singular kernel)
-      const cplx v = {acc.re * kInv4Pi, acc.im * kInv4Pi};
-      if constexpr (APPLY) {
-        const auto uj = constant_view(u) + 2 * (size_t)j;
-        const cplx t = cmul(v, {uj[0], uj[1]});
-        yi.re += t.re;
-        yi.im += t.im;
-      } else if (i_ok) {
-        store_entry(A.out, (long long)i + A.ld * (long long)j, v, skind, A.out_type, A.mode);
-      }
-      if (mirror) lds[wave][jj][lane] = make_double2(v.re, v.im);
+      finish(jj, sg, acc);
     }
+    if constexpr (GEN || APPLY)
+#pragma unroll 1
+      for (; near != 0; near &= near - 1) {
+        const int jj = __ffs(near) - 1, j = jbase + jj;  // per lane
+        const auto sg = trial_geo + (size_t)j * kGeoStride;
+        const auto sp = trial_vtx + (size_t)j * 12;
+        const double ny[3] = {sg[9], sg[10], sg[11]};
+        const double cs[3] = {sg[kGeoCentroid], sg[kGeoCentroid + 1], sg[kGeoCentroid + 2]};
+        const double D[3] = {ct[0] - cs[0], ct[1] - cs[1], ct[2] - cs[2]};
+        const double t[2][3] = {{tv[0], tv[1], tv[2]}, {tv[4], tv[5], tv[6]}};  // (td may be scaled)
+        const double d[2][3] = {{sp[0], sp[1], sp[2]}, {sp[4], sp[5], sp[6]}};
+        const double kappa = HELM ? fabs(A.k) : 0.0;
+        double kR = 0.0;
+        cplx e = {1.0, 0.0}, M[1][1];
+        if constexpr (CENTRED) e = pair_phase(ct, cs, kappa, &kR);
+        near_pair_sum<OP, HELM, CENTRED, false>(A, t, D, nx, ny, d, kappa, kR, M);
+        finish(jj, sg, scaled(M[0][0], tjx * sg[12], e));
+      }
     if (APPLY && mirror) {
       __syncthreads();
       // lane = (trial cell of the chunk, group of ch test cells); the start within the group is
