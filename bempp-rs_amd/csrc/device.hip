@@ -734,6 +734,9 @@ size_t max_tile_lds(int device) {
   return (size_t)bytes;
 }
 
+// Largest block of complex sums that the mixed-precision tiles with a P1 side take.
+constexpr size_t kMixedTileLds = 62 * 1024;
+
 // Tile coordinates (tile row = test block, tile column = trial block) for the
 // P0 x P0 kernel: all tiles, or the upper triangle a <= b when symmetric.
 // Cached per device and shape for the life of the process.
@@ -1192,7 +1195,8 @@ void assemble_device(const Assembler& a, const FunctionSpace& trial, const Funct
         const int nta = (R.n_test + dev::kTile - 1) / dev::kTile, ntb = (R.n_trial + dev::kTile - 1) / dev::kTile;
         int ntiles = 0;
         const int2* tiles = tile_list(P.device, nta, ntb, sym, &ntiles);
-        if (P.mixed)
+        // (blocks of many DOFs, as of meshes numbered in rows, are in FP64 whatever the precision asked for)
+        if (P.mixed && (size_t)tb->max_nd * sb->max_nd * sizeof(double2) <= kMixedTileLds)
           launch_mixed_lds(a.op, a.kind == kHelmholtz, P.tier, P.Q, dim3(ntiles), P.stream, R, tiles, sym ? 1 : 0,
                            tile_split(ntiles, kSplitP1), lds, P.near, P.near_segs, P.nsegs);
         else
