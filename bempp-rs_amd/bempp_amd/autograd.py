@@ -34,7 +34,9 @@ class BilinearForm(torch.autograd.Function):
         points, u, v = ctx.saved_tensors
         asm, space = ctx.assembler, ctx.space
         gn = complex(g.detach().cpu().item())
-        space.grid.set_points(_np(points).astype(np.float64))
+        p = _np(points).astype(np.float64)
+        if not np.array_equal(p, space.grid.points):  # moved since the forward pass
+            space.grid.set_points(p)
         grad_points = grad_u = grad_v = None
         if ctx.needs_input_grad[0]:
             G = asm.shape_gradient(space, space, _np(u), _np(v))

@@ -86,7 +86,7 @@ struct Grid {
   int cell_nv(int64_t c) const { return general() && types[c] == kQuadrilateral ? 4 : 3; }
   int64_t vertex(int64_t c, int m) const { return general() ? cell_verts[cell_off[c] + m] : cells[3 * c + m]; }
   // Same topology, new coordinates. Device data that depend on the topology alone (vertex ids,
-  // adjacent pairs) stay; so do all of them when the coordinates are the present ones.
+  // adjacent pairs) stay.
   void set_points(const double* pts);
 
   std::mutex cache_mutex;
