@@ -1531,9 +1531,9 @@ struct Prepared {
 };
 
 // stream: the launch stream; NULL selects the assembler's own stream unless caller_stream
-// is set (then NULL is the null stream).
+// is set (then NULL is the null stream). regular = false: without the regular rule's data of the cells.
 Prepared prepare(const Assembler& a, const FunctionSpace& trial, const FunctionSpace& test, void* out,
-                 void* stream, bool caller_stream = false);
+                 void* stream, bool caller_stream = false, bool regular = true);
 // The P0 x P0 tiles of a prepared assembly and the workgroups to split each over.
 const int2* p0_tile_list(const Prepared& P, bool symmetric, int* ntiles, int* split);
 // y += A_adjacent u (transpose: A_adjacent^T u) on P.stream; P0 spaces, u and y complex128.
