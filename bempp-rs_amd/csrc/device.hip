@@ -779,12 +779,16 @@ int tile_split(int ntiles, int most) {
 template <int OP, bool HELM, int CENTRED>
 void launch_q(int mode, int Q, dim3 grid, hipStream_t s, const dev::RegularArgs& A, const int2* tiles, int sym,
               int split, size_t lds) {
-  const dim3 parts(grid.x * split);
   constexpr int GC = CENTRED == 2 ? 1 : CENTRED;
-#define BEMPP_LAUNCH(QQ)                                                                                \
-  if (mode == 1) dev::regular_p0_tiled<QQ, OP, HELM, CENTRED><<<parts, 256, 0, s>>>(A, tiles, sym, split);       \
-  else if (mode == 2) dev::regular_tiled_lds<QQ, OP, HELM, CENTRED><<<parts, 256, lds, s>>>(A, tiles, sym, split); \
-  else dev::regular_kernel<QQ, OP, HELM, GC><<<grid, 256, 0, s>>>(A);
+#define BEMPP_LAUNCH(QQ)                                                                                        \
+  if (mode == 0) dev::regular_kernel<QQ, OP, HELM, GC><<<grid, 256, 0, s>>>(A);                                 \
+  else                                                                                                          \
+    in_launches(grid.x, [&](long long first, unsigned n) {                                                      \
+      if (mode == 1)                                                                                            \
+        dev::regular_p0_tiled<QQ, OP, HELM, CENTRED><<<n * split, 256, 0, s>>>(A, tiles + first, sym, split);   \
+      else                                                                                                      \
+        dev::regular_tiled_lds<QQ, OP, HELM, CENTRED><<<n * split, 256, lds, s>>>(A, tiles + first, sym, split); \
+    });
   switch (kernel_q(Q)) {
     case 1: BEMPP_LAUNCH(1); break;
     case 3: BEMPP_LAUNCH(3); break;

@@ -453,15 +453,16 @@ void apply(const Assembler& a, const FunctionSpace& trial, const FunctionSpace& 
   HIP_CHECK_G(hipGetLastError());
   int ntiles = 0, split = 1;
   const int2* tiles = p0_tile_list(P, symmetric, &ntiles, &split);
-  if (ntiles > 0) {
-    const dim3 grid((unsigned)ntiles * split);
-    const int sym = symmetric ? 1 : 0;
-    if (a.kind == kLaplace) launch_apply<false, 0>(P.Q, a.op, grid, s, P.R, tiles, sym, split, du, dy);
-    else if (P.tier == 2) launch_apply<true, 2>(P.Q, a.op, grid, s, P.R, tiles, sym, split, du, dy);
-    else if (P.tier == 1) launch_apply<true, 1>(P.Q, a.op, grid, s, P.R, tiles, sym, split, du, dy);
-    else if (P.tier == 3) launch_apply<true, 3>(P.Q, a.op, grid, s, P.R, tiles, sym, split, du, dy);
-    else launch_apply<true, 0>(P.Q, a.op, grid, s, P.R, tiles, sym, split, du, dy);
-  }
+  const int sym = symmetric ? 1 : 0;
+  in_launches(ntiles, [&](long long first, unsigned n) {
+    const dim3 grid(n * split);
+    const int2* t = tiles + first;
+    if (a.kind == kLaplace) launch_apply<false, 0>(P.Q, a.op, grid, s, P.R, t, sym, split, du, dy);
+    else if (P.tier == 2) launch_apply<true, 2>(P.Q, a.op, grid, s, P.R, t, sym, split, du, dy);
+    else if (P.tier == 1) launch_apply<true, 1>(P.Q, a.op, grid, s, P.R, t, sym, split, du, dy);
+    else if (P.tier == 3) launch_apply<true, 3>(P.Q, a.op, grid, s, P.R, t, sym, split, du, dy);
+    else launch_apply<true, 0>(P.Q, a.op, grid, s, P.R, t, sym, split, du, dy);
+  });
   apply_adjacent(a, P, du, dy, transpose);
   HIP_CHECK_G(hipMemcpyAsync(hy.data(), dy, hy.size() * sizeof(double), hipMemcpyDeviceToHost, s));
   HIP_CHECK_G(hipStreamSynchronize(s));

@@ -1476,6 +1476,14 @@ struct GradientInputs {
   void* stream;
 };
 
+// Launches f(first, n) over `count` workgroups in runs of at most 2^21: a launch has to stay below 2^32
+// threads, of which a workgroup has up to 1024.
+template <typename F>
+void in_launches(long long count, F f) {
+  constexpr long long kMost = 1LL << 21;
+  for (long long first = 0; first < count; first += kMost) f(first, (unsigned)(count - first < kMost ? count - first : kMost));
+}
+
 struct Assembler;      // core.hpp
 struct FunctionSpace;  // core.hpp
 

@@ -61,6 +61,7 @@ struct PotentialArgs {
   int out_type;
   int mode;                // kStore or kAccumulate (one writer per entry), or kAtomic (cells once)
   int parts;               // workgroups the cells are split over (1 with blocks)
+  long long first;         // first group (of a DOF block and a block of points) of the launch
 };
 
 // TIER (Helmholtz): 0 full argument reduction per point pair; 1, 2, 3: |k| t rad <= 0.5 / 0.25 /
@@ -74,7 +75,7 @@ __global__ void __launch_bounds__(1024) potential_kernel(const PotentialArgs A) 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int part = blockIdx.x % A.parts;
-  const long long group = blockIdx.x / A.parts;
+  const long long group = A.first + blockIdx.x / A.parts;
   const long long block = group / A.npblocks;
   const long long t = (group - block * A.npblocks) * 64 + lane;
   const bool ok = t < A.np;
@@ -265,14 +266,16 @@ void assemble_potential_device(const Assembler& a, const FunctionSpace& space, c
       }
     }
   }
-  if (groups * P.parts > INT32_MAX) throw Error("too many evaluation points");
-  const dim3 g((unsigned)(groups * P.parts));
   const bool helm = a.kind == kHelmholtz;
   // |k (r - R)| <= |k| t rad (with a margin for the rounding of r and R)
   const double bound = std::fabs(a.k) * in.rule_radius * in.max_radius * (1.0 + 1e-12);
   const int tier = !helm || !dev::scalable(a.k, in.max_radius) ? 0 : bound <= 0.25 ? 2 : bound <= 0.5 ? 1 : bound <= 1.5 ? 3 : 0;
-  if (a.op == kSL) launch_potential<0>(in.Q, helm, tier, in.nb, g, s, P);
-  else launch_potential<1>(in.Q, helm, tier, in.nb, g, s, P);
+  in_launches(groups, [&](long long first, unsigned n) {
+    P.first = first;
+    const dim3 g(n * P.parts);  // (parts > 1 only where that gives at most 8192)
+    if (a.op == kSL) launch_potential<0>(in.Q, helm, tier, in.nb, g, s, P);
+    else launch_potential<1>(in.Q, helm, tier, in.nb, g, s, P);
+  });
   HIP_CHECK_P(hipGetLastError());
 }
 
