@@ -915,7 +915,8 @@ regular_tiled_lds(const RegularArgs A, const int2* __restrict__ tiles, int symme
 // Args: RegularArgs, possibly qualified with the constant address space (batched
 // launches read each item's arguments in place, with scalar loads).
 // APPLY: the entries are not stored but applied, y += A u (u, y complex128; atomics): the lane's
-// row in a register, the mirrored rows by summing a chunk's entries over the lanes.
+// row in a register, the mirrored rows by summing a chunk's products over the lanes. Entries of adjacent
+// pairs are left out, not applied as zeros (which would turn an infinite entry of u into NaN).
 template <int Q, int OP, bool HELM, int CENTRED, int CH = kChunk, int NW = 4, bool APPLY = false, typename Args>
 __device__ __forceinline__ void p0_tile(Args& A, const int2 tile, int symmetric,
                                         double2 (&lds)[NW][CH][kTile], int split = 1, int part = 0,
@@ -968,7 +969,10 @@ __device__ __forceinline__ void p0_tile(Args& A, const int2 tile, int symmetric,
                 "chunk must divide the trial cells of a wavefront");
   const int tpw = kTile / NW / split;  // trial cells per wavefront
   const int ch = min(CH, tpw), chs = __builtin_ctz(ch);
-  cplx yi = {0.0, 0.0};
+  cplx yi = {0.0, 0.0}, ui = {0.0, 0.0};
+  if constexpr (APPLY) {
+    if (mirror) ui = {u[2 * (size_t)il], u[2 * (size_t)il + 1]};
+  }
   for (int c = 0; c < tpw; c += ch) {
     const int jbase = tile.y * kTile + (part * NW + wave) * tpw + c;
     unsigned near = 0;  // the lane's near trial cells of the chunk (the orbit sums of the dense tiles take r^2 by terms at
@@ -986,10 +990,14 @@ __device__ __forceinline__ void p0_tile(Args& A, const int2 tile, int symmetric,
         const cplx t = cmul(v, {uj[0], uj[1]});
         yi.re += t.re;
         yi.im += t.im;
-      } else if (i_ok) {
-        store_entry(A.out, (long long)i + A.ld * (long long)j, v, skind, A.out_type, A.mode);
+        if (mirror) {
+          const cplx m = cmul(v, ui);
+          lds[wave][jj][lane] = make_double2(m.re, m.im);
+        }
+      } else {
+        if (i_ok) store_entry(A.out, (long long)i + A.ld * (long long)j, v, skind, A.out_type, A.mode);
+        if (mirror) lds[wave][jj][lane] = make_double2(v.re, v.im);
       }
-      if (mirror) lds[wave][jj][lane] = make_double2(v.re, v.im);
     };
     // the sum of group_pair_sum or near_pair_sum, times f and e^{i kappa R}
     auto scaled = [&](cplx m, double f, cplx e) {
@@ -1044,7 +1052,8 @@ __device__ __forceinline__ void p0_tile(Args& A, const int2 tile, int symmetric,
           acc = p0_pair_orbit<Q, OP, HELM, 0>(td, tau2g, twc, sp, D, R2, nx, ny, A.k, 0.0);
         }
       }
-      finish(jj, sg, acc);
+      if (!APPLY || !left) finish(jj, sg, acc);
+      else if (mirror) lds[wave][jj][lane] = make_double2(0.0, 0.0);
     }
     if constexpr (GEN || APPLY)
 #pragma unroll 1
@@ -1076,9 +1085,8 @@ __device__ __forceinline__ void p0_tile(Args& A, const int2 tile, int symmetric,
         const int ic = tile.x * kTile + col;
         if (ic < A.n_test) {
           const double2 val = lds[wave][row][col];
-          const cplx t = cmul({val.x, val.y}, {u[2 * (size_t)ic], u[2 * (size_t)ic + 1]});
-          sum.re += t.re;
-          sum.im += t.im;
+          sum.re += val.x;
+          sum.im += val.y;
         }
       }
       for (int off = ch; off < 64; off <<= 1) {
