@@ -314,12 +314,14 @@ __device__ __forceinline__ T load_uniform(const T* p) {
   return v;
 }
 
+// Centroid distance R of a cell pair from R^2; 0 for cells that cross at their centroids.
+__device__ __forceinline__ double centroid_distance(double R2) { return R2 * rsqrt_nr(fmax(R2, 1e-280)); }
+
 // e^{ikR} for the centroid distance R of a cell pair (CENTRED Helmholtz pairs).
 __device__ __forceinline__ cplx pair_phase(const double* ct, const double* cs, double k, double* kR) {
   const double dx = ct[0] - cs[0], dy = ct[1] - cs[1], dz = ct[2] - cs[2];
   const double R2 = dx * dx + dy * dy + dz * dz;
-  const double R = R2 * rsqrt_nr(R2);
-  *kR = k * R;
+  *kR = k * centroid_distance(R2);
   cplx e;
   sincos_cw(*kR, &e.im, &e.re);
   return e;
@@ -452,7 +454,7 @@ __device__ __forceinline__ void p1_cell_pair(const RegularArgs& A, const P1TestC
   double kR = 0.0;
   cplx e = {1.0, 0.0};
   if constexpr (TIER > 0) {
-    kR = kappa * (R2 * rsqrt_nr(R2));
+    kR = kappa * centroid_distance(R2);
     sincos_cw(kR, &e.im, &e.re);
   }
   cplx M[NB][NB];
