@@ -258,23 +258,21 @@ __global__ void __launch_bounds__(256) cells_regular_kernel(const CellsArgs A) {
             for (int d = 0; d < 3; ++d) cp[u][a][d] = P[12 + 3 * a + d];
         }
       }
-      {
-        for (int q = 0; q < nq; ++q) {
-          const auto Q = Qj + (size_t)q * kRec;
-          const double xq[3] = {Q[0], Q[1], Q[2]}, nq3[3] = {Q[4], Q[5], Q[6]};
-          double phq[NBS], cq[NBS][3];
+      for (int q = 0; q < nq; ++q) {
+        const auto Q = Qj + (size_t)q * kRec;
+        const double xq[3] = {Q[0], Q[1], Q[2]}, nq3[3] = {Q[4], Q[5], Q[6]};
+        double phq[NBS], cq[NBS][3];
 #pragma unroll
-          for (int b = 0; b < NBS; ++b) {
-            phq[b] = NBS == 1 ? 1.0 : Q[8 + b];
-            if constexpr (OP == 3)
+        for (int b = 0; b < NBS; ++b) {
+          phq[b] = NBS == 1 ? 1.0 : Q[8 + b];
+          if constexpr (OP == 3)
 #pragma unroll
-              for (int d = 0; d < 3; ++d) cq[b][d] = Q[12 + 3 * b + d];
-          }
-#pragma unroll
-          for (int u = 0; u < PP; ++u)
-            add_point_pair<OP, HELM, NBT, NBS, TIER>(xp[u], np[u], php[u], cp[u], xq, nq3, phq, cq, wJp[u] * Q[3],
-                                                     wp[u] * Q[7], A.k, M, kR);
+            for (int d = 0; d < 3; ++d) cq[b][d] = Q[12 + 3 * b + d];
         }
+#pragma unroll
+        for (int u = 0; u < PP; ++u)
+          add_point_pair<OP, HELM, NBT, NBS, TIER>(xp[u], np[u], php[u], cp[u], xq, nq3, phq, cq, wJp[u] * Q[3],
+                                                   wp[u] * Q[7], A.k, M, kR);
       }
     };
     if constexpr (NBT * NBS <= 4) {

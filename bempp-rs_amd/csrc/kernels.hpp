@@ -100,9 +100,7 @@ struct RegularArgs {
 struct SingularArgs {
   const int4* pairs;        // test cell, trial cell, shared count, permutation code
   int npairs;
-  const double* rule;       // 5 arrays of rule_total: test xi0, test xi1, trial xi0, trial xi1, weight
-  const double* rule_aos;   // the same rule, one record of 6 per point: a0 a1 b0 b1 w pad
-  int rule_total;
+  const double* rule_aos;   // one record of 6 per rule point: a0 a1 b0 b1 w pad (test, trial coordinates, weight)
   int rule_off[4];          // indexed by shared count 1..3
   int rule_n[4];
   const double* test_geo;
