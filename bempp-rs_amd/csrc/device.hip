@@ -67,6 +67,7 @@ struct DeviceSpaceCache {
   int* pot_cells = nullptr;
   int* pot_ldof = nullptr;
   int pot_nblocks = 0;
+  int64_t pot_entries = -1;  // cells listed, with repetitions
 };
 
 void drop_device_geometry(DeviceGridCache* c) {
@@ -1346,6 +1347,29 @@ void assemble_singular_csr(const Assembler& a, const FunctionSpace& trial, const
 }
 
 // ---- potential (off-surface) operators ----
+// The distinct blocks of a cell's DOFs, in the order of its DOFs.
+static int cell_dof_blocks(const FunctionSpace& s, int64_t cell, int64_t (&blk)[3]) {
+  int n = 0;
+  for (int a = 0; a < s.nb; ++a) {
+    const int64_t b = s.dofs[cell * s.nb + a] / kPotentialDofs;
+    if (std::find(blk, blk + n, b) == blk + n) blk[n++] = b;
+  }
+  return n;
+}
+
+// Evaluations of the space's cells by blocks: the cells that the blocks list, with repetitions.
+static int64_t potential_entries(FunctionSpace& s, int device) {
+  space_dofs(s, device);
+  std::lock_guard<std::mutex> lk(s.cache_mutex);
+  DeviceSpaceCache* c = s.device_cache.at(device);
+  if (c->pot_entries < 0) {
+    int64_t blk[3], n = 0;
+    for (int64_t cell = 0; cell < s.grid->nc(); ++cell) n += cell_dof_blocks(s, cell, blk);
+    c->pot_entries = n;
+  }
+  return c->pot_entries;
+}
+
 // DOF blocks of a space for the potential kernel (PotentialInputs): each DOF belongs to one
 // block, so the block's workgroups sum its entries over the listed cells and write each once.
 static const DeviceSpaceCache* potential_blocks(FunctionSpace& s, int device) {
@@ -1357,18 +1381,9 @@ static const DeviceSpaceCache* potential_blocks(FunctionSpace& s, int device) {
   const int nb = s.nb;
   const int64_t nblk = (s.size + kPotentialDofs - 1) / kPotentialDofs;
   std::vector<int> off(nblk + 1, 0);
-  // the distinct blocks of a cell's DOFs, in the order of its DOFs
-  auto cell_blocks = [&](int64_t cell, int64_t (&blk)[3]) {
-    int n = 0;
-    for (int a = 0; a < nb; ++a) {
-      const int64_t b = s.dofs[cell * nb + a] / kPotentialDofs;
-      if (std::find(blk, blk + n, b) == blk + n) blk[n++] = b;
-    }
-    return n;
-  };
   int64_t blk[3];
   for (int64_t cell = 0; cell < nc; ++cell)
-    for (int m = cell_blocks(cell, blk) - 1; m >= 0; --m) ++off[blk[m] + 1];
+    for (int m = cell_dof_blocks(s, cell, blk) - 1; m >= 0; --m) ++off[blk[m] + 1];
   for (int64_t b = 0; b < nblk; ++b) off[b + 1] += off[b];
   // one upload: off, cells, ldof back to back
   const size_t ne = (size_t)off[nblk];
@@ -1377,7 +1392,7 @@ static const DeviceSpaceCache* potential_blocks(FunctionSpace& s, int device) {
   int* cells = lists.data() + nblk + 1;
   int* ldof = cells + ne;
   for (int64_t cell = 0; cell < nc; ++cell)
-    for (int m = cell_blocks(cell, blk) - 1; m >= 0; --m) {
+    for (int m = cell_dof_blocks(s, cell, blk) - 1; m >= 0; --m) {
       const int e = at[blk[m]]++;
       cells[e] = (int)cell;
       for (int a = 0; a < nb; ++a) {
@@ -1419,14 +1434,24 @@ PotentialInputs potential_inputs(const Assembler& a, const FunctionSpace& space_
   P.ngroups = (int)rg.groups.size();
   P.wc = rg.wc;
   P.wc_trial = space.nb == 3 ? rg.wc / 3.0 : rg.wc;
-  // DOF blocks pay where cells share DOFs, but a cell at their borders is evaluated for each: with few
-  // workgroups and many rule points (evaluations, not atomics, then take the time) the cells are
-  // taken once, with atomics. P1, 16 points, blocks / cells once: Laplace single layer, 306 workgroups of
-  // blocks, 34.6 / 31 us, 480: 40 / 36.5, 3807: 193 / 280; Helmholtz double layer, 84: 48.5 / 30; 6 points, 90:
-  // 24.4 / 27. Nothing is built while the stream is captured: blocks only if an earlier call did.
+  // DOF blocks pay where cells share DOFs, but a cell at their borders is evaluated for each: 1.57 times on an
+  // icosphere, 2.48 times in random cell order. Many evaluations, or few workgroups, cost more than the atomics of
+  // taking the cells once. P1, 16 points, blocks / cells once: Laplace single layer, 306 workgroups of blocks,
+  // 34.6 / 31 us, 480: 40 / 36.5, 3807: 193 / 280; Helmholtz double layer, 84: 48.5 / 30; 6 points, 90: 24.4 / 27.
+  // By evaluations of rule points a cell, 5120 cells, 10007 points: Laplace single layer, 25: 555 / 986, 40:
+  // 880 / 973 (1000 points: 111 / 99), 58: 1120 / 1050, 92: 1760 / 1028; Helmholtz double layer, 58: 3246 / 3999,
+  // 92: 5104 / 3993; 50 points: Helmholtz double layer, 21 workgroups, 9: 23 / 16, 81 workgroups, 9: 23 / 25, 15:
+  // 33 / 24, 321 workgroups, 15: 64 / 78; Laplace, 15: 31 / 26. Nothing is built while the stream is captured:
+  // blocks only if an earlier call did.
   const long long pblocks = (npoints + 63) / 64, dblocks = (space.size + kPotentialDofs - 1) / kPotentialDofs;
+  const long long groups = pblocks * dblocks;
   const bool shared_dofs = space.size < (int64_t)space.nb * grid.nc();
-  bool blocks = shared_dofs && (P.Q <= dev::kMaxQ || pblocks * dblocks >= 512);
+  bool blocks = shared_dofs && (P.Q <= dev::kMaxQ || groups >= 512);
+  if (blocks) {
+    const double evaluations = (double)potential_entries(space, device) / (double)grid.nc() * P.Q;
+    blocks = evaluations <= (a.kind == kHelmholtz ? std::min(80.0, groups / 4.0 - 10.0)
+                                                  : std::min(35.0, std::max(10.0, groups / 24.0)));
+  }
   if (blocks && stream) {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     HIP_CHECK(hipStreamIsCapturing((hipStream_t)stream, &capture));
