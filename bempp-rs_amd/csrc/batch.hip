@@ -166,11 +166,6 @@ void check_versions(const Batch& b) {
       throw Error("a grid of the batch changed after the batch was built; build a new batch");
 }
 
-long long batch_tiles(int ncells, bool symmetric) {
-  const long long n = (ncells + dev::kTile - 1) / dev::kTile;
-  return symmetric ? n * (n + 1) / 2 : n * n;
-}
-
 hipStream_t own_stream(Batch& b) {
   if (!b.stream) HIP_CHECK_B(hipStreamCreateWithFlags(&b.stream, hipStreamNonBlocking));
   return b.stream;
@@ -240,24 +235,6 @@ Batch* batch_new(const std::vector<const Assembler*>& asms, const std::vector<co
   for (size_t i = 0; i < n; ++i) {
     if (b->mixed && tiers[i] == 3) tiers[i] = 0;
     centred[i] = tiers[i] == 1 || tiers[i] == 2 ? 1 : 0;
-  }
-  // A tier of few tiles joins the next more general one in use (2, 1, 3, 0: each holds for the items of those
-  // before it): the launches follow each other, and one below two rounds of the default workgroups costs more than
-  // its cheaper sine and cosine saves. 18 ellipsoids of 320 and 1280 cells, 3-point rule, tiles 90 / 420 / 210 / 1305
-  // of tiers 0 to 3: 521 -> 499 us
-  if (!b->mixed && b->kind == kHelmholtz) {
-    long long tiles[4] = {0, 0, 0, 0};
-    for (size_t i = 0; i < n; ++i) tiles[tiers[i]] += batch_tiles(R[i].n_test, b->symmetric);
-    const int general[4] = {2, 1, 3, 0};
-    for (int g = 0; g < 3; ++g) {
-      const int from = general[g];
-      int to = g + 1;
-      while (to < 4 && tiles[general[to]] == 0) ++to;
-      if (tiles[from] == 0 || tiles[from] >= 2LL * b->blocks_per_cu * b->cus || to == 4) continue;
-      std::replace(tiers.begin(), tiers.end(), from, general[to]);
-      tiles[general[to]] += tiles[from];
-      tiles[from] = 0;
-    }
   }
   // tile lists in two orders, each grouped by phase mode (non-centred items first)
   std::stable_sort(size_order.begin(), size_order.end());
