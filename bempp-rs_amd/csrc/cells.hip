@@ -396,8 +396,9 @@ __global__ void __launch_bounds__(256) point_views_kernel(const double* __restri
 // share each trial point read from LDS (broadcasts; 48-byte records, so that a barrier covers
 // 32 cells of 16 points), and the test points are read coalesced. Cells near each other take r^2 from
 // the differences X - o_q (group_near).
-// Bound by FP64 VALU issue, 22 + rsq (Helmholtz tier 2) instructions per point pair.
-// Helmholtz, 5400 cells of 16 points, tier 1, with the adjacent pairs: 4.94 -> 4.58 ms.
+// Bound by FP64 VALU issue (95 % busy), 22 + rsq (Helmholtz tier 2) instructions per point pair.
+// Helmholtz, 5400 cells of 16 points, tier 1, with the adjacent pairs: 4.99 -> 4.86 ms, where two runs of one
+// side differ by 5 %.
 constexpr int kSlStage = 512;  // records staged per workgroup (24 KB)
 
 template <bool HELM, int TIER>
@@ -1026,7 +1027,7 @@ void assemble_cells_device(const Assembler& a, const FunctionSpace& trial, const
   const int bx = (A.n_test + 255) / 256;
   // trial cells per workgroup: few enough for 32768 workgroups (half of them idle by symmetry), so that
   // small grids fill the card and the last workgroups are short. Single layer, 16 points, at least
-  // four cells and 16384 workgroups / so: 384 cells 205 / 171 us, 864: 455 / 399, 5400: 4.93 / 4.84 ms;
+  // four cells and 16384 workgroups / so: 384 cells 205 / 171 us, 864: 455 / 399;
   // P1 hypersingular, 1176 cells: 2.39 / 2.26 ms
   long long chunk = ((long long)bx * A.n_trial + 32767) / 32768;
   chunk = std::max(1LL, std::min(64LL, chunk));

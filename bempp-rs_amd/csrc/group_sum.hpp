@@ -16,13 +16,13 @@
 namespace bempp_amd {
 namespace dev {
 
-// Bound by FP64 VALU issue; a point pair of the 6-point rule on P1 costs 14.5 (Laplace double
-// layer) to 30 (Helmholtz) instructions with its share of everything per test point and cell
+// Bound by FP64 VALU issue (88 to 96 % busy); a point pair of the 6-point rule on P1 costs 14.5 (Laplace
+// double layer) to 30 (Helmholtz) instructions with its share of everything per test point and cell
 // pair, against 22 and 43 with point coordinates, trial points in SGPRs (which spilled) and
-// test points re-read per trial cell (which kept the vector L1 busy). Whole assemblies:
-// Helmholtz hypersingular P1, 20480 cells, 6 points: 19.5 -> 12.1 ms; Laplace double layer P1, 19110
-// cells: 12.0 -> 8.5 ms; Laplace single layer P1, 5120 cells, 16 points: 3.13 -> 1.55 ms;
-// Helmholtz single layer P0, 5120 cells, 37 points: 18.0 -> 15.2 ms. Loops over a run-time number
+// test points re-read per trial cell (which kept the vector L1 busy). Whole assemblies, near pairs included:
+// Helmholtz hypersingular P1, 20480 cells, 6 points: 19.4 -> 11.8 ms; Laplace double layer P1, 19110
+// cells: 12.0 -> 8.6 ms; Laplace single layer P1, 5120 cells, 16 points: 3.12 -> 1.64 ms;
+// Helmholtz single layer P0, 5120 cells, 37 points: 17.7 -> 16.1 ms. Loops over a run-time number
 // of groups two at a time measured the same.
 
 // Fields of a group's record in the device table (RegularArgs::groups, kGroupStride doubles).

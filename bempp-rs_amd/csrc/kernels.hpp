@@ -841,7 +841,7 @@ __device__ __forceinline__ void flush_tile(const Args& A, const double* acc, int
 // output with one global atomic. symmetric (single layer / hypersingular on one space):
 // tiles a <= b only; an off-diagonal tile also adds its entries at the transposed place.
 // Dynamic LDS: (test block DOFs) x (trial block DOFs) doubles, twice that for complex kernels.
-// Waves per SIMD: Laplace 4 (at most 127 VGPRs); Helmholtz 3 with 4 to 10 VGPRs spilled (the
+// Waves per SIMD: Laplace 4 (at most 128 VGPRs); Helmholtz 3 with up to 24 VGPRs spilled (the
 // hypersingular kernel unconstrained took 266 and ran 17.7 ms at 20480 cells against 12.1), 2
 // for rules of a run-time point count (3 would spill 55 to 69).
 // ---------------------------------------------------------------------------

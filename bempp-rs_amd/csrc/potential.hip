@@ -6,16 +6,16 @@
 // scalar loads. Where cells share DOFs it also owns kPotentialDofs consecutive DOFs, whose entries it
 // alone writes: P1 entries are summed in LDS at [DOF][point] (lane = point, so the LDS adds of a
 // wavefront never collide) and each is written once, 64 consecutive points a column. A cell at the
-// border of two DOF blocks is evaluated for both (about 1.5 times the cells of a 32-vertex patch):
-// cheaper than adding every cell's three entries to the output with global FP64 atomics, which ran at
-// ~83 G/s and bounded the kernel, except for few workgroups and many rule points. Without shared
+// border of two DOF blocks is evaluated for both (1.6 times where the cell order has locality, 2.5 in
+// random order): cheaper than adding every cell's three entries to the output with global FP64 atomics, which
+// ran at ~83 G/s and bounded the kernel, except for many evaluations or few workgroups. Without shared
 // DOFs the entries are stored where they are computed, 64 consecutive points a column.
 //
 // The phase is taken relative to kR, R the distance of the point from the cell's centroid:
 // |k (r - R)| <= |k| |y - c| for every point y of the cell wherever the evaluation point is, so the
 // small-argument tiers hold by the cells' size alone and e^{ikR} is applied once per (point, cell).
 //
-// Bound by FP64 VALU issue. Helmholtz single layer, P1, 10007 points, 5120 cells, 6-point rule,
+// Bound by FP64 VALU issue (92 % busy). Helmholtz single layer, P1, 10007 points, 5120 cells, 6-point rule,
 // complex128: 3.83 ms with the atomics and a full phase reduction per point pair, 0.69 ms so.
 #include <hip/hip_runtime.h>
 
